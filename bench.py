@@ -615,7 +615,8 @@ def main() -> int:
 
     import torch
 
-    from turboexl3_amd import api
+    from turboexl3_amd import api, build
+    build.ensure_built()
     if not torch.cuda.is_available():
         print("bench.py: no GPU visible", file=sys.stderr)
         return 2

@@ -14,10 +14,9 @@ def pytest_configure(config):
 
 def pytest_sessionstart(session):
     """The tests load the in-tree library and call it only; a tree where nothing is built yet gets built once."""
-    from turboexl3_amd import _lib, build
+    from turboexl3_amd import build
 
-    if not os.path.exists(_lib.LIB_PATH):
-        build.build()
+    build.ensure_built()
 
 
 def has_gpu() -> bool:

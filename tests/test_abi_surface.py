@@ -13,8 +13,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 @pytest.fixture(scope="module")
 def lib():
     from turboexl3_amd import _lib, build
-    if not os.path.exists(_lib.LIB_PATH):
-        build.build()
+    build.ensure_built()
     return _lib.lib()
 
 

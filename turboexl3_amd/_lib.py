@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libturboexl3_hip.so")
@@ -162,27 +163,29 @@ def lib() -> C.CDLL:
 
 
 _binding = None
+_binding_lock = threading.Lock()  # threads whose first calls meet load the extension once
 
 
 def binding():
     """The native side of `turboexl3_amd.api` (csrc/t3_torch.cpp): torch tensors in, a torch tensor out, one call of the C
     ABI between. Raises if it has not been built."""
     global _binding
-    if _binding is None:
-        import importlib.machinery
-        import importlib.util
+    with _binding_lock:
+        if _binding is None:
+            import importlib.machinery
+            import importlib.util
 
-        import torch  # noqa: F401  (its libraries come first: the binding links them)
+            import torch  # noqa: F401  (its libraries come first: the binding links them)
 
-        lib()
-        if not os.path.exists(TORCH_LIB_PATH):
-            raise RuntimeError(f"{TORCH_LIB_PATH} is missing: build it with `python -m turboexl3_amd.build`")
-        loader = importlib.machinery.ExtensionFileLoader("_t3_torch", TORCH_LIB_PATH)
-        spec = importlib.util.spec_from_file_location("_t3_torch", TORCH_LIB_PATH, loader=loader)
-        mod = importlib.util.module_from_spec(spec)
-        loader.exec_module(mod)
-        _binding = mod
-    return _binding
+            lib()
+            if not os.path.exists(TORCH_LIB_PATH):
+                raise RuntimeError(f"{TORCH_LIB_PATH} is missing: build it with `python -m turboexl3_amd.build`")
+            loader = importlib.machinery.ExtensionFileLoader("_t3_torch", TORCH_LIB_PATH)
+            spec = importlib.util.spec_from_file_location("_t3_torch", TORCH_LIB_PATH, loader=loader)
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+            _binding = mod
+        return _binding
 
 
 def error_name(status: int) -> str:

@@ -123,8 +123,19 @@ def release_engines() -> None:
     _lib.lib().t3_release_engines()
 
 
-_native = _lib.binding()
-_native.bind(_workspaces, _workspace, T3Error)
+class _Unbound:
+    """Stands for the native binding until the first call needs it: importing this package loads no library, so that what
+    builds it, and the modules that run without a GPU, can be imported from a tree where nothing is built yet."""
+
+    def __getattr__(self, name):
+        global _native
+        native = _lib.binding()
+        native.bind(_workspaces, _workspace, T3Error)
+        _native = native  # from here on a call looks its function up in the extension module itself
+        return getattr(native, name)
+
+
+_native = _Unbound()
 
 
 def _plan_dict(p) -> dict:

@@ -128,5 +128,11 @@ def build(force: bool = False, jobs: int = 8) -> str:
     return LIB
 
 
+def ensure_built() -> None:
+    """Builds where a library is missing: for programs that load what is there and build only a tree where nothing is."""
+    if not (os.path.exists(LIB) and os.path.exists(TORCH_LIB)):
+        build()
+
+
 if __name__ == "__main__":
     print(build(force="--force" in sys.argv))
