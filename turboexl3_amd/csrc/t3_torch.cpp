@@ -35,7 +35,10 @@ void check(int32_t status) {
     if (status != T3_OK) refuse(status);
 }
 
-// A tensor's descriptor, and the tensor that owns its bytes (a contiguous copy where the caller's is not).
+// A tensor's descriptor, and the tensor that owns its bytes (a contiguous copy where the caller's is not). It is held until
+// the call is over whoever else holds it: an attribute may be computed and have no other owner, and another thread may
+// replace a bank's while this one runs without the interpreter lock; memory freed meanwhile would be handed out again as
+// the call's own output or workspace.
 struct Arg {
     t3_array a;
     at::Tensor keep;
@@ -75,12 +78,8 @@ void read(PyObject* o, Arg* out) {
         PyErr_SetString(PyExc_ValueError, "turboexl3_amd runs on device tensors only");
         throw PythonError{};
     }
-    if (t.is_contiguous()) {
-        describe(t, dtype, &out->a);  // the caller's own reference keeps it
-    } else {
-        out->keep = t.contiguous();
-        describe(out->keep, dtype, &out->a);
-    }
+    out->keep = t.is_contiguous() ? t : t.contiguous();
+    describe(out->keep, dtype, &out->a);
 }
 
 // An attribute of a Python object, owned for the scope.
@@ -114,7 +113,7 @@ void read_proj(PyObject* bank, PyObject* name, t3_proj* p, at::Tensor* keep) {
     PyObject* const names[3] = {s_trellis, s_suh, s_svh};
     t3_array* const arrays[3] = {&p->trellis, &p->suh, &p->svh};
     for (int i = 0; i < 3; ++i) {
-        const Attr t(proj.p, names[i]);  // the bank keeps it past this scope
+        const Attr t(proj.p, names[i]);
         Arg a;
         read(t.p, &a);
         *arrays[i] = a.a;
@@ -137,8 +136,10 @@ t3_stream stream_of(PyObject* o) {
 }
 
 struct Workspace {
+    at::Tensor keep;
     void* p;
     size_t bytes;
+    explicit Workspace(const at::Tensor& t) : keep(t), p(t.data_ptr()), bytes(static_cast<size_t>(t.numel())) {}
 };
 
 // The thread's workspace on x's device, grown by the Python side where it is too small. The dict owns it and stays the
@@ -158,14 +159,13 @@ Workspace workspace_for(PyObject* x, size_t need) {
     if (!ws && PyErr_Occurred()) throw PythonError{};
     if (ws) {
         const at::Tensor& t = THPVariable_Unpack(ws);
-        if (static_cast<size_t>(t.numel()) >= need) return {t.data_ptr(), static_cast<size_t>(t.numel())};
+        if (static_cast<size_t>(t.numel()) >= need) return Workspace(t);
     }
     const Attr dev(x, s_device);
     PyObject* made = PyObject_CallFunction(g_workspace, "On", dev.p, static_cast<Py_ssize_t>(need));
     if (!made) throw PythonError{};
-    const at::Tensor& t = THPVariable_Unpack(made);
-    const Workspace w{t.data_ptr(), static_cast<size_t>(t.numel())};
-    Py_DECREF(made);  // the dict holds it
+    const Workspace w(THPVariable_Unpack(made));
+    Py_DECREF(made);
     return w;
 }
 
