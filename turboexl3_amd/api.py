@@ -6,6 +6,7 @@ libturboexl3_hip.so through the C ABI, which the calls of a serving loop reach t
 (csrc/t3_torch.cpp) and the calls around it (plans, loading, self-tests) through ctypes."""
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import threading
 from dataclasses import dataclass
@@ -93,6 +94,17 @@ def _stream_ptr(stream) -> int:
     return s.cuda_stream
 
 
+def _on(stream, t):
+    """The scope in which `stream` is the current one of t's device: what a call makes beside its launches (contiguous copies,
+    outputs, a cleared workspace) is then made in that stream's order. None: the current stream as it is."""
+    if stream is None or not isinstance(t, torch.Tensor) or not t.is_cuda:  # the last two: the call refuses t
+        return contextlib.nullcontext()
+    if not isinstance(stream, torch.cuda.Stream):  # any object with a `cuda_stream` will do
+        raw = stream.cuda_stream
+        stream = torch.cuda.ExternalStream(raw, device=t.device) if raw else torch.cuda.default_stream(t.device)
+    return torch.cuda.stream(stream)
+
+
 _workspaces: dict = {}
 
 
@@ -102,6 +114,8 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     key = (device.type, device.index, threading.get_ident())
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
+        if ws is not None and ws.is_cuda:
+            ws.record_stream(torch.cuda.current_stream(device))  # the stream its last call, ordered before this one, ended on
         # zero-filled once: the head of a workspace holds the fused launches' arrival counters
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
@@ -168,12 +182,13 @@ def linear(x, trellis, suh, svh, dec: Decode = Decode.mul1, stream=None) -> torc
 def linear_static(x, trellis, suh, svh, dec: Decode = Decode.mul1, stream=None, out=None) -> torch.Tensor:
     """`linear` at decode rows through the entry point that allocates nothing: its scratch is the library's own device
     array (16 MiB a GPU). `out`: the caller's y (this harness allocates one otherwise; the C call never does)."""
-    ax, at, asu, asv = _arr(x), _arr(trellis), _arr(suh), _arr(svh)
-    y = out if out is not None else torch.empty(*x.shape[:-1], trellis.shape[1] * 16, dtype=x.dtype, device=x.device)
-    ay = _arr(y)
-    _check(_lib.lib().t3_linear_static(_stream_ptr(stream), C.byref(ax), C.byref(at), C.byref(asu), C.byref(asv), dec.c(),
-                                       C.byref(ay)))
-    return y
+    with _on(stream, x):
+        ax, at, asu, asv = _arr(x), _arr(trellis), _arr(suh), _arr(svh)
+        y = out if out is not None else torch.empty(*x.shape[:-1], trellis.shape[1] * 16, dtype=x.dtype, device=x.device)
+        ay = _arr(y)
+        _check(_lib.lib().t3_linear_static(_stream_ptr(stream), C.byref(ax), C.byref(at), C.byref(asu), C.byref(asv), dec.c(),
+                                           C.byref(ay)))
+        return y
 
 
 def linear_static_reset(stream=None) -> None:
@@ -188,13 +203,14 @@ def linear_chain(x, trellis, suh, svh, dec: Decode = Decode.mul1, stream=None) -
 
 def dequant(trellis, dec: Decode = Decode.mul1, stream=None) -> torch.Tensor:
     """W_hat f16 [in, out]: format.reconstructInner on the device, bit-exact."""
-    at = _arr(trellis)
-    if trellis.dim() != 3:
-        raise T3Error(1)
-    w = torch.empty(trellis.shape[0] * 16, trellis.shape[1] * 16, dtype=torch.float16, device=trellis.device)
-    aw = _arr(w)
-    _check(_lib.lib().t3_dequant(_stream_ptr(stream), C.byref(at), dec.c(), C.byref(aw)))
-    return w
+    with _on(stream, trellis):
+        at = _arr(trellis)
+        if trellis.dim() != 3:
+            raise T3Error(1)
+        w = torch.empty(trellis.shape[0] * 16, trellis.shape[1] * 16, dtype=torch.float16, device=trellis.device)
+        aw = _arr(w)
+        _check(_lib.lib().t3_dequant(_stream_ptr(stream), C.byref(at), dec.c(), C.byref(aw)))
+        return w
 
 
 def linear_resident(x, w_hat, suh, svh, stream=None) -> torch.Tensor:
@@ -206,20 +222,21 @@ def unrot_weight(trellis, suh, svh, dec: Decode = Decode.mul1, dtype=torch.bfloa
                  stream=None):
     """The un-rotated weight W_std [in, out] in `dtype` (dense.unrotWeight), or written into columns col0.. of `into`
     (a join: one [in, N] array, its members side by side). Returns (w_std, nonfinite count)."""
-    L = _lib.lib()
-    at = _arr(trellis)
-    if trellis.dim() != 3:
-        raise T3Error(1)
-    in_f, out_f = trellis.shape[0] * 16, trellis.shape[1] * 16
-    w = into if into is not None else torch.empty(in_f, out_f, dtype=dtype, device=trellis.device)
-    need = C.c_size_t(0)
-    _check(L.t3_unrot_workspace_bytes(C.byref(at), C.byref(need)))
-    ws = _workspace(trellis.device, need.value)
-    bad = torch.zeros(1, dtype=torch.int32, device=trellis.device)
-    asu, asv, aw = _arr(suh), _arr(svh), _arr(w)
-    _check(L.t3_unrot_weight(_stream_ptr(stream), C.byref(at), C.byref(asu), C.byref(asv), dec.c(), C.byref(aw), col0,
-                             bad.data_ptr(), ws.data_ptr(), ws.numel()))
-    return w, int(bad.item())
+    with _on(stream, trellis):
+        L = _lib.lib()
+        at = _arr(trellis)
+        if trellis.dim() != 3:
+            raise T3Error(1)
+        in_f, out_f = trellis.shape[0] * 16, trellis.shape[1] * 16
+        w = into if into is not None else torch.empty(in_f, out_f, dtype=dtype, device=trellis.device)
+        need = C.c_size_t(0)
+        _check(L.t3_unrot_workspace_bytes(C.byref(at), C.byref(need)))
+        ws = _workspace(trellis.device, need.value)
+        bad = torch.zeros(1, dtype=torch.int32, device=trellis.device)
+        asu, asv, aw = _arr(suh), _arr(svh), _arr(w)
+        _check(L.t3_unrot_weight(_stream_ptr(stream), C.byref(at), C.byref(asu), C.byref(asv), dec.c(), C.byref(aw), col0,
+                                 bad.data_ptr(), ws.data_ptr(), ws.numel()))
+        return w, int(bad.item())
 
 
 def linear_unrot(x, w_std, col0: int = 0, cols=None, stream=None) -> torch.Tensor:
@@ -320,26 +337,28 @@ def moe_fused_shared_routed(x, bank: Bank, logits, k: int, dec: Decode, shared_b
     slots = rows * k
     pad = lambda b: (b + 255) & ~255
     tail = need.value - pad(slots * 4) - pad(slots * 2) - 256
-    inds = ws[tail:tail + slots * 4].view(torch.int32).reshape(rows, k).clone()
-    scores = ws[tail + pad(slots * 4):tail + pad(slots * 4) + slots * 2].view(x.dtype).reshape(rows, k).clone()
-    if gate_vec is None:
-        return y, inds, scores
-    glogit = ws[need.value - 256:need.value - 256 + rows * 2].view(torch.bfloat16).clone()
-    return y, inds, scores, glogit
+    with _on(stream, x):
+        inds = ws[tail:tail + slots * 4].view(torch.int32).reshape(rows, k).clone()
+        scores = ws[tail + pad(slots * 4):tail + pad(slots * 4) + slots * 2].view(x.dtype).reshape(rows, k).clone()
+        if gate_vec is None:
+            return y, inds, scores
+        glogit = ws[need.value - 256:need.value - 256 + rows * 2].view(torch.bfloat16).clone()
+        return y, inds, scores, glogit
 
 
 def moe_glm(x, bank: Bank, inds, dec: Decode, limit: int = 0, stream=None, fill: float = 0.0) -> torch.Tensor:
     """The routed experts under GLM's rounding profile: x bf16 [B, S, D] -> f32 [B, S, K, D], a slot's own output each
     (a skipped slot keeps `fill`)."""
-    L = _lib.lib()
-    ax, ai = _arr(x), _arr(inds)
-    cb, _keep = _cbank(bank)
-    ws = _moe_workspace(L, ax, cb, ai, x.device)
-    y = torch.full((x.shape[0], x.shape[1], inds.shape[2], x.shape[2]), fill, dtype=torch.float32, device=x.device)
-    ay = _arr(y)
-    _check(L.t3_moe_glm(_stream_ptr(stream), C.byref(ax), C.byref(cb), C.byref(ai), dec.c(), int(limit), C.byref(ay),
-                        ws.data_ptr(), ws.numel()))
-    return y
+    with _on(stream, x):
+        L = _lib.lib()
+        ax, ai = _arr(x), _arr(inds)
+        cb, _keep = _cbank(bank)
+        ws = _moe_workspace(L, ax, cb, ai, x.device)
+        y = torch.full((x.shape[0], x.shape[1], inds.shape[2], x.shape[2]), fill, dtype=torch.float32, device=x.device)
+        ay = _arr(y)
+        _check(L.t3_moe_glm(_stream_ptr(stream), C.byref(ax), C.byref(cb), C.byref(ai), dec.c(), int(limit), C.byref(ay),
+                            ws.data_ptr(), ws.numel()))
+        return y
 
 
 # ---- device self-tests -------------------------------------------------------------------------------------

@@ -13,6 +13,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <optional>
+
 #include "../../include/turboexl3_hip.h"
 
 namespace {
@@ -127,13 +129,36 @@ void read_bank(PyObject* o, BankArg* out) {
     read_proj(o, s_down, &out->b.down, out->keep + 6);
 }
 
-t3_stream stream_of(PyObject* o) {
-    if (o == Py_None) return c10::hip::getCurrentHIPStream().stream();
-    const Attr s(o, s_cuda_stream);
-    void* p = PyLong_AsVoidPtr(s.p);
-    if (!p && PyErr_Occurred()) throw PythonError{};
-    return p;
-}
+// The stream a call runs on: the caller's, or the current one. A given stream is the current one of x's device for the
+// scope, so that whatever the call makes on the way, the contiguous copies, the output and a workspace that is cleared, is
+// made in that stream's order and not beside it.
+class CallStream {
+public:
+    CallStream(PyObject* stream, PyObject* x) {
+        if (stream == Py_None) return;
+        const Attr s(stream, s_cuda_stream);
+        void* p = PyLong_AsVoidPtr(s.p);
+        if (!p && PyErr_Occurred()) throw PythonError{};
+        given_ = true;
+        raw_ = p;
+        if (!THPVariable_Check(x) || !THPVariable_Unpack(x).is_cuda()) return;  // read() refuses it
+        const c10::DeviceIndex device = THPVariable_Unpack(x).device().index();
+        const c10::hip::HIPStream now = c10::hip::getCurrentHIPStream(device);
+        if (now.stream() == static_cast<hipStream_t>(p)) return;
+        before_ = now;
+        c10::hip::setCurrentHIPStream(c10::hip::getStreamFromExternal(static_cast<hipStream_t>(p), device));
+    }
+    ~CallStream() {
+        if (before_) c10::hip::setCurrentHIPStream(*before_);
+    }
+    CallStream(const CallStream&) = delete;
+    t3_stream get() const { return given_ ? raw_ : c10::hip::getCurrentHIPStream().stream(); }
+
+private:
+    bool given_ = false;
+    void* raw_ = nullptr;
+    std::optional<c10::hip::HIPStream> before_;
+};
 
 struct Workspace {
     at::Tensor keep;
@@ -214,6 +239,7 @@ void unlocked(F&& f) {
 PyObject* py_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 8)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[6], v[0]);
         Arg x, t, suh, svh, bias;
         read(v[0], &x);
         read(v[1], &t);
@@ -224,7 +250,7 @@ PyObject* py_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
         const t3_decode dec = read_decode(v[5]);
         size_t need = 0;
         check(t3_linear_workspace_bytes(&x.a, &t.a, dec, &need));
-        const t3_stream stream = stream_of(v[6]);
+        const t3_stream stream = on.get();
         const bool chain = v[7] == Py_True;
         t3_array ay;
         at::TensorBase y = new_output(v[0], t.a.shape[1] * 16, &ay);
@@ -241,6 +267,7 @@ PyObject* py_linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* py_linear_resident(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 5)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[4], v[0]);
         Arg x, w, suh, svh;
         read(v[0], &x);
         read(v[1], &w);
@@ -248,7 +275,7 @@ PyObject* py_linear_resident(PyObject*, PyObject* const* v, Py_ssize_t n) {
         read(v[3], &svh);
         size_t need = 0;
         check(t3_linear_resident_workspace_bytes(&x.a, &w.a, &need));
-        const t3_stream stream = stream_of(v[4]);
+        const t3_stream stream = on.get();
         t3_array ay;
         at::TensorBase y = new_output(v[0], w.a.shape[1], &ay);
         const Workspace ws = workspace_for(v[0], need);
@@ -261,12 +288,13 @@ PyObject* py_linear_resident(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* py_linear_unrot(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 6)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[4], v[0]);
         Arg x, w;
         read(v[0], &x);
         read(v[1], &w);
         const int64_t col0 = as_long(v[2]), cols = as_long(v[3]);
         if (cols < 0) refuse(T3_BadExl3Shape);
-        const t3_stream stream = stream_of(v[4]);
+        const t3_stream stream = on.get();
         size_t need = 0;
         if (v[5] == Py_True) check(t3_linear_unrot_workspace_bytes(&x.a, &w.a, col0, cols, &need));
         t3_array ay;
@@ -287,6 +315,7 @@ enum MoeEntry : long { kMoe, kClamped, kSwiglu, kWithShared, kSharedExpert };
 PyObject* py_moe(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 10)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[9], v[1]);
         const long entry = as_long(v[0]);
         Arg x, inds, scores, add;
         BankArg bank, shared;
@@ -300,7 +329,7 @@ PyObject* py_moe(PyObject*, PyObject* const* v, Py_ssize_t n) {
         const int32_t i0 = static_cast<int32_t>(as_long(v[6])), i1 = static_cast<int32_t>(as_long(v[7]));
         size_t need = 0;
         check(t3_moe_workspace_bytes(&x.a, &bank.b, &inds.a, entry == kSharedExpert ? &shared.b : nullptr, &need));
-        const t3_stream stream = stream_of(v[9]);
+        const t3_stream stream = on.get();
         t3_array ay;
         at::TensorBase y = new_output(v[1], -1, &ay);
         const Workspace ws = workspace_for(v[1], need);
@@ -327,6 +356,7 @@ PyObject* py_moe(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* py_moe_fused_shared(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 9)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[8], v[0]);
         Arg x, inds, scores, tab, logit;
         BankArg bank, shared;
         read(v[0], &x);
@@ -339,7 +369,7 @@ PyObject* py_moe_fused_shared(PyObject*, PyObject* const* v, Py_ssize_t n) {
         check(t3_moe_workspace_bytes(&x.a, &bank.b, &inds.a, &shared.b, &need));
         read(v[6], &tab);
         read(v[7], &logit);
-        const t3_stream stream = stream_of(v[8]);
+        const t3_stream stream = on.get();
         t3_array ay;
         at::TensorBase y = new_output(v[0], -1, &ay);
         const Workspace ws = workspace_for(v[0], need);
@@ -355,6 +385,7 @@ PyObject* py_moe_fused_shared(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* py_moe_fused_shared_routed(PyObject*, PyObject* const* v, Py_ssize_t n) {
     if (!arity(n, 10)) return nullptr;
     return guarded([&] {
+        const CallStream on(v[9], v[0]);
         Arg x, logits, tab, logit, gate;
         BankArg bank, shared;
         read(v[0], &x);
@@ -368,7 +399,7 @@ PyObject* py_moe_fused_shared_routed(PyObject*, PyObject* const* v, Py_ssize_t n
         read(v[6], &tab);
         if (v[7] != Py_None) read(v[7], &logit);
         if (v[8] != Py_None) read(v[8], &gate);
-        const t3_stream stream = stream_of(v[9]);
+        const t3_stream stream = on.get();
         t3_array ay;
         at::TensorBase y = new_output(v[0], -1, &ay);
         const Workspace ws = workspace_for(v[0], need);

@@ -7,7 +7,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from .api import _arr, _stream_ptr, _workspace
+from .api import _arr, _on, _stream_ptr, _workspace
 
 NAME = "turboexl3"  # table/table.zig:27
 
@@ -69,19 +69,20 @@ def load_bank(block: _lib.Block, trellis, suh, svh, in_dim: int = 0) -> _lib.Wei
 
 
 def matmul(w: _lib.Weight, x: torch.Tensor, stream=None) -> torch.Tensor:
-    L = _lib.lib()
-    ax = _arr(x)
-    need = C.c_size_t(0)
-    st = L.t3_table_matmul_workspace_bytes(C.byref(w), C.byref(ax), C.byref(need))
-    if st != 0:
-        raise Refused(_lib.VERDICT_UNSUPPORTED, _lib.error_name(st))
-    y = torch.empty(*x.shape[:-1], w.w.shape[1] * 16, dtype=x.dtype, device=x.device)
-    ay = _arr(y)
-    ws = _workspace(x.device, need.value)
-    buf = C.create_string_buffer(128)
-    _verdict(L.t3_table_matmul(_stream_ptr(stream), C.byref(w), C.byref(ax), C.byref(ay), ws.data_ptr(), ws.numel(), buf,
-                               len(buf)), buf)
-    return y
+    with _on(stream, x):
+        L = _lib.lib()
+        ax = _arr(x)
+        need = C.c_size_t(0)
+        st = L.t3_table_matmul_workspace_bytes(C.byref(w), C.byref(ax), C.byref(need))
+        if st != 0:
+            raise Refused(_lib.VERDICT_UNSUPPORTED, _lib.error_name(st))
+        y = torch.empty(*x.shape[:-1], w.w.shape[1] * 16, dtype=x.dtype, device=x.device)
+        ay = _arr(y)
+        ws = _workspace(x.device, need.value)
+        buf = C.create_string_buffer(128)
+        _verdict(L.t3_table_matmul(_stream_ptr(stream), C.byref(w), C.byref(ax), C.byref(ay), ws.data_ptr(), ws.numel(), buf,
+                                   len(buf)), buf)
+        return y
 
 
 def moe() -> None:
@@ -91,15 +92,16 @@ def moe() -> None:
 
 def swiglu(gate: _lib.Weight, up: _lib.Weight, down: _lib.Weight, x, inds, scores, limit: int = 0,
            verify_rows: bool = False, stream=None) -> torch.Tensor:
-    L = _lib.lib()
-    ax, ai, asc = _arr(x), _arr(inds), _arr(scores)
-    need = C.c_size_t(0)
-    buf = C.create_string_buffer(128)
-    y = torch.empty_like(x)
-    ay = _arr(y)
-    st = L.t3_table_swiglu_workspace_bytes(C.byref(gate), C.byref(up), C.byref(down), C.byref(ax), C.byref(ai), C.byref(need))
-    ws = _workspace(x.device, need.value if st == 0 else 0)
-    _verdict(L.t3_table_swiglu(_stream_ptr(stream), C.byref(gate), C.byref(up), C.byref(down), C.byref(ax), C.byref(ai),
-                               C.byref(asc), limit, int(verify_rows), C.byref(ay), ws.data_ptr(), ws.numel(), buf, len(buf)),
-             buf)
-    return y
+    with _on(stream, x):
+        L = _lib.lib()
+        ax, ai, asc = _arr(x), _arr(inds), _arr(scores)
+        need = C.c_size_t(0)
+        buf = C.create_string_buffer(128)
+        y = torch.empty_like(x)
+        ay = _arr(y)
+        st = L.t3_table_swiglu_workspace_bytes(C.byref(gate), C.byref(up), C.byref(down), C.byref(ax), C.byref(ai), C.byref(need))
+        ws = _workspace(x.device, need.value if st == 0 else 0)
+        _verdict(L.t3_table_swiglu(_stream_ptr(stream), C.byref(gate), C.byref(up), C.byref(down), C.byref(ax), C.byref(ai),
+                                   C.byref(asc), limit, int(verify_rows), C.byref(ay), ws.data_ptr(), ws.numel(), buf, len(buf)),
+                 buf)
+        return y
