@@ -34,3 +34,59 @@ def test_rows_equal_their_decode_calls(hidden, inter, rows, topk, decode, dtype)
     rms = want.square().mean().sqrt()
     step = 2.0 ** (-7 if dtype == torch.bfloat16 else -9)
     assert bool(((y - want).abs() <= step * want.abs() + 2e-2 * rms).all()), float((y - want).abs().max() / rms)
+
+
+def case(t3, hidden, inter, rows, topk, n=64, experts=9, unit_scales=False):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(hidden + inter)
+
+    def scales(width):
+        v = torch.randn(experts, width, device="cuda", generator=g)
+        return torch.where(v < 0, -1.0, 1.0) if unit_scales else v
+
+    def proj(in_f, out_f):
+        return t3.Proj(torch.randint(-32768, 32768, (experts, in_f // 16, out_f // 16, n), dtype=torch.int16, device="cuda",
+                                     generator=g),
+                       scales(in_f).half(), (scales(out_f) * in_f ** -0.5).half())
+
+    bank = t3.Bank(proj(hidden, inter), proj(hidden, inter), proj(inter, hidden))
+    x = torch.randn(1, rows, hidden, device="cuda", generator=g).half()
+    inds = torch.rand(rows, experts, device="cuda", generator=g).topk(topk).indices.to(torch.int32)[None].contiguous()
+    inds[0, ::5, 0] = -1  # skipped
+    return x, bank, inds, torch.rand(1, rows, topk, device="cuda", generator=g)
+
+
+@pytest.mark.parametrize("hidden,inter", [(128, 384), (640, 1152), (2432, 128), (2176, 2304)])
+@pytest.mark.parametrize("decode", ["mcg", "mul1"])
+def test_a_rows_bytes_do_not_depend_on_how_many_waves_share_its_blocks(hidden, inter, decode):
+    """The fewer the positions, the more waves share one's blocks: up to one a block, or 16, 8, 4 of a workgroup where its block
+    sums are added up. Rows of one long call against shorter calls' at every step, skipped slots among them."""
+    from turboexl3_amd import api as t3
+    dec = getattr(t3.Decode, decode)
+    x, bank, inds, scores = case(t3, hidden, inter, 2900, 3)
+    whole = t3.moe(x, bank, inds, scores, dec)  # 2175 groups of four positions
+    assert bool(torch.isfinite(whole).all())
+    for rows in (17, 40, 341, 342, 1300, 1366):
+        part = t3.moe(x[:, :rows].contiguous(), bank, inds[:, :rows].contiguous(), scores[:, :rows].contiguous(), dec)
+        assert torch.equal(part, whole[:, :rows]), rows
+
+
+@pytest.mark.parametrize("hidden,inter", [(65664, 128), (128, 65664), (665600, 128)])
+def test_block_sums_of_very_wide_rows(hidden, inter):
+    """More 128-blocks than their sums have LDS at a time (and, the last, than a workgroup has at all): f16 rows against their
+    decode calls, which add the same sums up elsewhere."""
+    from turboexl3_amd import api as t3
+    dec = t3.Decode.mul1
+    x, bank, inds, scores = case(t3, hidden, inter, 18, 2, n=16, experts=3, unit_scales=True)
+    y = t3.moe(x, bank, inds, scores, dec).float()
+    want = torch.cat([t3.moe(x[:, r:r + 1].contiguous(), bank, inds[:, r:r + 1].contiguous(), scores[:, r:r + 1].contiguous(), dec)
+                      for r in range(4)], 1).float()
+    # Two chains that round to f16 at the same points and differ in the order of their f32 sums alone: a value may round to the
+    # next f16 (2^-10 of it at most). An element's own three roundings (the down sums, the finish, the output) move it by 3 such
+    # steps; the six of the gate, up and hidden values reach it through the 128-blocks' transforms and the sums as noise of at
+    # most sqrt(6) 2^-10 of the row's rms, and five times that is the largest of the 2.7 million values looked at. (Scales of one
+    # size: the noise of a column is as large as its scale.) A total that misses any of its blocks is off by whole rms.
+    rms = want.square().mean(-1, keepdim=True).sqrt()
+    step = 2.0 ** -10
+    worst = ((y[:, :4] - want).abs() - 3 * step * want.abs()).div(5 * 6 ** 0.5 * step * rms).max()
+    assert float(worst) <= 1.0, float(worst)

@@ -396,25 +396,40 @@ __global__ void __launch_bounds__(256) pf_place(const MoeLaunch a) {
 // One wave takes kPfUnit 128-blocks (adjacent ones of a row, or one of each of four sorted positions), 16 lanes a block and 8
 // adjacent elements a lane (t3_stages.hpp, "four 128-blocks a wave"): every load and store is 16 bytes a lane, and a block's transform
 // is ~20 vector-ALU operations a lane (the one-block-a-wave form of the decode kernels spends ~100: these kernels were
-// bound by it). Four waves a workgroup; grid ceil(units / 4). Blocks past the row's last one load the last block and
-// store nothing. Every array these kernels touch starts 16-byte aligned (the host checks the caller's).
+// bound by it). Where a wave's blocks are a row's: four waves a workgroup, grid ceil(units / 4), and blocks past the row's last
+// one load the last block and store nothing. Every array these kernels touch starts 16-byte aligned (the host checks the caller's).
 
 constexpr uint32_t kPfUnit = 4;
 
 __device__ __forceinline__ uint32_t wave_unit() { return blockIdx.x * 4u + (threadIdx.x >> 6); }
 
-// The prepare and the mid stage: a workgroup takes four positions, each of its waves all four of them, 16 lanes a position and
-// every fourth 128-block. A position's place in the order, its expert and its row (three loads one behind the other) are
-// looked up once for all of a wave's blocks, a block's loads go out before the one in front of it is worked on, and four
-// positions of one expert (they are sorted by it) read its scales together. A wave of four adjacent blocks of one position
-// took 183 us for the prepare of 16,384 positions of 7168 (the looking up, and its stores of four bytes a lane), this form 128
-// (it writes 470 MB, about 100 us); the mid stage of 2048 wide, bound by its vector arithmetic, 80 and 79. Where a position's block sums are wanted in order (MUL1's deferred map), the waves leave theirs in LDS and a
-// thread a position adds them up.
-inline dim3 position_grid(uint32_t positions) { return dim3((positions + 3u) / 4u); }
-__device__ __forceinline__ float ordered_total(const float* sums, uint32_t nb) {
-    float acc = 0.0f;
-    for (uint32_t b = 0; b < nb; ++b) acc += sums[b];
-    return acc;
+// The prepare and the mid stage: a wave takes four positions, 16 lanes a position and one 128-block a turn. A position's place
+// in the order, its expert and its row (three loads one behind the other) are looked up once for all of a wave's blocks, a
+// block's loads go out before the one in front of it is worked on, and four positions of one expert (they are sorted by it)
+// read its scales together.
+//
+// How many waves share the blocks of four positions (stage_waves): four where the positions alone fill the GPU, more the fewer
+// they are, up to a wave a block. With four always, a short prompt's few waves walked their blocks one behind the other: us for
+// 7168 x 2048 at 17 tokens top-2 / 64 top-8 / 128 top-10 / 512 top-8, the prepare 14.2 / 15.5 / 20.2 / 31.4 -> 3.2 / 6.8 / 13.0 /
+// 28.4, the mid stage 8.4 / 8.6 / 12.0 / 22.1 -> 4.0 / 4.9 / 8.0 / 20.3 (at half as many waves 13.4 and 30.3, 8.7 and 21.8).
+// Which waves make a workgroup: in the prepare, waves of adjacent blocks of the same positions (its stores, most of its bytes,
+// then go out a kilobyte a position at a time: 32,768 positions of 4096, 149 -> 134 us); in the mid stage, whose rows may be
+// three or five blocks, waves of adjacent positions and the same blocks, none of which is idle (13,280 positions of 640
+// 22.7 -> 21.8, 16,384 of 384 18.7 -> 17.1).
+// TOTALS: MUL1's deferred map wants a position's block sums added up in order. All the waves of its blocks are then one
+// workgroup, which leaves the sums in LDS, kPfSumBlocks blocks at a time, and a thread a position adds them up. 16 waves where
+// positions are few (17 tokens top-2 of 7168 x 2048: the prepare 16.3 -> 9.6, the mid stage 8.9 -> 6.8), four where they are many
+// (more wait longer for one another: 13,280 positions of 640 wide, the mid stage 24 with four, 33 with eight).
+constexpr uint32_t kPfSumBlocks = 512;
+__host__ __device__ inline uint32_t sum_chunk(uint32_t nb) { return nb < kPfSumBlocks ? nb : kPfSumBlocks; }
+inline uint32_t stage_waves(uint32_t positions, uint32_t nb, bool totals) {
+    const uint32_t groups = (positions + 3u) / 4u;
+    const uint32_t most = totals ? (groups <= 256u ? 16u : groups < 1024u ? 8u : 4u) : (groups >= 2048u ? 4u : 8192u / groups);
+    return most < nb ? most : nb;
+}
+
+__device__ __forceinline__ void add_ordered(float& acc, const float* sums, uint32_t n) {
+    for (uint32_t b = 0; b < n; ++b) acc += sums[b];
 }
 
 // a lane's eight activations as they lie in memory
@@ -448,13 +463,15 @@ struct ActWords {
     }
 };
 
-// totals (null: not wanted): a position's sum of its blocks' sums, gate and up: f32 [2][positions]; dynamic LDS: the blocks'
-// sums, [2][4][blocks]
-template <int DT, int PROF>
-__global__ void __launch_bounds__(256) pf_prep(const MoeLaunch a, float* totals, uint32_t positions) {
-    extern __shared__ float block_sums[];
-    __shared__ __attribute__((aligned(16))) uint32_t tr[4][256];
+// Grid (position groups, parts / 4), 256 threads; TOTALS: (position groups), 64 x parts threads. totals: a position's sum of its
+// blocks' sums, gate and up: f32 [2][positions]. Dynamic LDS: 1 KB a wave for the pair-quad order, then TOTALS' block sums.
+template <int DT, int PROF, bool TOTALS>
+__global__ void __launch_bounds__(TOTALS ? 1024 : 256) pf_prep(const MoeLaunch a, float* totals, uint32_t positions, uint32_t parts) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t stage_mem[];
     const uint32_t nb = a.hidden / 128u, first = blockIdx.x * 4u, lane = threadIdx.x & 63u, q = lane & 15u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), chunk = TOTALS ? sum_chunk(nb) : nb;
+    uint32_t* tr = stage_mem + wave * 256u;
+    float* block_sums = reinterpret_cast<float*>(stage_mem + parts * 256u);  // [gate, up][4 positions][chunk]
     const uint32_t placed = a.counts[a.bank.experts + a.shared_slots + 1u];
     if (first >= placed) return;
     const uint32_t p1 = first + (lane >> 4);
@@ -476,40 +493,51 @@ __global__ void __launch_bounds__(256) pf_prep(const MoeLaunch a, float* totals,
         l.sc[0] = load8_words(suh_g, i);
         l.sc[1] = load8_words(suh_u, i);
     };
-    uint32_t b = threadIdx.x >> 6;
+    uint32_t b = TOTALS ? wave : blockIdx.y * 4u + wave;
     Loads next;
     if (b < nb) load(b, next);
-    while (b < nb) {
-        const Loads cur = next;
-        const uint32_t now = b;
-        b += 4u;
-        if (b < nb) load(b, next);
-        float xv[8];
-        cur.x.template values<PROF == 0>(xv);
-#pragma unroll
-        for (uint32_t proj = 0; proj < 2u; ++proj) {
-            float v[8], sum;
-            product8(xv, cur.sc[proj], v);
-            const uint4v hv = pair_quad_pieces(tr[threadIdx.x >> 6], lane, prep_row16(v, g16, sum, a.defer != 0));
-            if (totals && q == 0u) block_sums[(proj * 4u + (lane >> 4)) * nb + now] = sum;
-            if (!live) continue;
-            *reinterpret_cast<uint4v*>(reinterpret_cast<uint16_t*>(proj ? a.xu : a.xg) + orow + now * 128u + 8u * q) = hv;
-            if (PROF != 0 && a.defer && q == 0u) (proj ? a.su : a.sg)[static_cast<size_t>(pos) * nb + now] = sum;
-        }
-    }
-    if (!totals) return;
-    __syncthreads();
     const uint32_t t = threadIdx.x;
-    if (t < 8u && first + (t & 3u) < placed) totals[(t >> 2) * positions + first + (t & 3u)] = ordered_total(block_sums + t * nb, nb);
+    float total = 0.0f;
+    for (uint32_t from = 0; from < nb; from += chunk) {
+        const uint32_t to = nb - from > chunk ? from + chunk : nb;
+        while (b < to) {
+            const Loads cur = next;
+            const uint32_t now = b;
+            b += parts;
+            if (b < nb) load(b, next);
+            float xv[8];
+            cur.x.template values<PROF == 0>(xv);
+#pragma unroll
+            for (uint32_t proj = 0; proj < 2u; ++proj) {
+                float v[8], sum;
+                product8(xv, cur.sc[proj], v);
+                const uint4v hv = pair_quad_pieces(tr, lane, prep_row16(v, g16, sum, a.defer != 0));
+                if (TOTALS && q == 0u) block_sums[(proj * 4u + (lane >> 4)) * chunk + now - from] = sum;
+                if (!live) continue;
+                *reinterpret_cast<uint4v*>(reinterpret_cast<uint16_t*>(proj ? a.xu : a.xg) + orow + now * 128u + 8u * q) = hv;
+                if (PROF != 0 && a.defer && q == 0u) (proj ? a.su : a.sg)[static_cast<size_t>(pos) * nb + now] = sum;
+            }
+        }
+        if (!TOTALS) return;
+        __syncthreads();
+        if (t < 8u) add_ordered(total, block_sums + t * chunk, to - from);
+        if (to == nb) break;
+        __syncthreads();
+    }
+    if (t < 8u && first + (t & 3u) < placed) totals[(t >> 2) * positions + first + (t & 3u)] = total;
 }
 
 // gate and up finishes, the (clamped) SwiGLU, the down's prepare (routed_mid_block's statements)
-// totals: as the prepare's, of the down projection's input, f32 [positions]; dynamic LDS [4][blocks]
-template <int PROF>
-__global__ void __launch_bounds__(256) pf_mid(const MoeLaunch a, float* totals) {
-    extern __shared__ float block_sums[];
-    __shared__ __attribute__((aligned(16))) uint32_t tr[4][256];
-    const uint32_t nb = a.inter / 128u, first = blockIdx.x * 4u, lane = threadIdx.x & 63u, q = lane & 15u;
+// Grid (four position groups, parts), 256 threads; TOTALS: as the prepare. totals: as the prepare's, of the down projection's
+// input, f32 [positions]
+template <int PROF, bool TOTALS>
+__global__ void __launch_bounds__(TOTALS ? 1024 : 256) pf_mid(const MoeLaunch a, float* totals, uint32_t parts) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t stage_mem[];
+    const uint32_t nb = a.inter / 128u, lane = threadIdx.x & 63u, q = lane & 15u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), chunk = TOTALS ? sum_chunk(nb) : nb;
+    const uint32_t first = (TOTALS ? blockIdx.x : blockIdx.x * 4u + wave) * 4u;
+    uint32_t* tr = stage_mem + wave * 256u;
+    float* block_sums = reinterpret_cast<float*>(stage_mem + parts * 256u);  // [4 positions][chunk]
     const uint32_t placed = a.counts[a.bank.experts + a.shared_slots + 1u];
     if (first >= placed) return;
     const uint32_t p1 = first + (lane >> 4);
@@ -547,55 +575,62 @@ __global__ void __launch_bounds__(256) pf_mid(const MoeLaunch a, float* totals) 
         l.svu = load8_words(bank.up_svh, eo + i);
         l.sdn = load8_words(bank.down_suh, eo + i);
     };
-    uint32_t b = threadIdx.x >> 6;
+    uint32_t b = TOTALS ? wave : blockIdx.y;
     Loads next;
     if (b < nb) load(b, next);
-    while (b < nb) {
-        const Loads cur = next;
-        const uint32_t now = b;
-        b += 4u;
-        if (b < nb) load(b, next);
-        float gt[8], up[8], d[8], sum;
-        if constexpr (PROF == 0) {
-            unpack8(cur.zg[0], gt);
-            unpack8(cur.zu[0], up);
-            unpack8(finish_row16(gt, cur.svg, g16), gt);
-            unpack8(finish_row16(up, cur.svu, g16), up);
+    const uint32_t t = threadIdx.x;
+    float total = 0.0f;
+    for (uint32_t from = 0; from < nb; from += chunk) {
+        const uint32_t to = nb - from > chunk ? from + chunk : nb;
+        while (b < to) {
+            const Loads cur = next;
+            const uint32_t now = b;
+            b += parts;
+            if (b < nb) load(b, next);
+            float gt[8], up[8], d[8], sum;
+            if constexpr (PROF == 0) {
+                unpack8(cur.zg[0], gt);
+                unpack8(cur.zu[0], up);
+                unpack8(finish_row16(gt, cur.svg, g16), gt);
+                unpack8(finish_row16(up, cur.svu, g16), up);
 #pragma unroll
-            for (uint32_t r = 0; r < 8u; ++r) d[r] = swiglu_clamped(gt[r], up[r], a.limit, a.clamp_at);
-            unpack8(pack8(d), d);  // rounded to f16
-        } else {
-#pragma unroll
-            for (uint32_t r = 0; r < 8u; ++r) {
-                gt[r] = __builtin_bit_cast(float, static_cast<uint32_t>(cur.zg[r >> 2][r & 3u]));
-                up[r] = __builtin_bit_cast(float, static_cast<uint32_t>(cur.zu[r >> 2][r & 3u]));
-            }
-            if (a.defer) {
+                for (uint32_t r = 0; r < 8u; ++r) d[r] = swiglu_clamped(gt[r], up[r], a.limit, a.clamp_at);
+                unpack8(pack8(d), d);  // rounded to f16
+            } else {
 #pragma unroll
                 for (uint32_t r = 0; r < 8u; ++r) {
-                    gt[r] = __builtin_fmaf(gt[r], mul1_a(), mul1_b() * xg);
-                    up[r] = __builtin_fmaf(up[r], mul1_a(), mul1_b() * xu);
+                    gt[r] = __builtin_bit_cast(float, static_cast<uint32_t>(cur.zg[r >> 2][r & 3u]));
+                    up[r] = __builtin_bit_cast(float, static_cast<uint32_t>(cur.zu[r >> 2][r & 3u]));
                 }
-            }
-            float sv[8];
-            unpack8(cur.svg, sv);
-            finish_row16_glm(gt, sv, g16, true);
-            unpack8(cur.svu, sv);
-            finish_row16_glm(up, sv, g16, true);
+                if (a.defer) {
 #pragma unroll
-            for (uint32_t r = 0; r < 8u; ++r) d[r] = swiglu_glm(gt[r], up[r], a.limit);
+                    for (uint32_t r = 0; r < 8u; ++r) {
+                        gt[r] = __builtin_fmaf(gt[r], mul1_a(), mul1_b() * xg);
+                        up[r] = __builtin_fmaf(up[r], mul1_a(), mul1_b() * xu);
+                    }
+                }
+                float sv[8];
+                unpack8(cur.svg, sv);
+                finish_row16_glm(gt, sv, g16, true);
+                unpack8(cur.svu, sv);
+                finish_row16_glm(up, sv, g16, true);
+#pragma unroll
+                for (uint32_t r = 0; r < 8u; ++r) d[r] = swiglu_glm(gt[r], up[r], a.limit);
+            }
+            product8(d, cur.sdn, d);
+            const uint4v hv = pair_quad_pieces(tr, lane, prep_row16(d, g16, sum, a.defer != 0));
+            if (TOTALS && q == 0u) block_sums[(lane >> 4) * chunk + now - from] = sum;
+            if (!live) continue;
+            *reinterpret_cast<uint4v*>(reinterpret_cast<uint16_t*>(a.hd) + qo + now * 128u + 8u * q) = hv;
+            if (PROF != 0 && a.defer && q == 0u) a.hs[static_cast<size_t>(pos) * nb + now] = sum;
         }
-        product8(d, cur.sdn, d);
-        const uint4v hv = pair_quad_pieces(tr[threadIdx.x >> 6], lane, prep_row16(d, g16, sum, a.defer != 0));
-        if (totals && q == 0u) block_sums[(lane >> 4) * nb + now] = sum;
-        if (!live) continue;
-        *reinterpret_cast<uint4v*>(reinterpret_cast<uint16_t*>(a.hd) + qo + now * 128u + 8u * q) = hv;
-        if (PROF != 0 && a.defer && q == 0u) a.hs[static_cast<size_t>(pos) * nb + now] = sum;
+        if (!TOTALS) return;
+        __syncthreads();
+        if (t < 4u) add_ordered(total, block_sums + t * chunk, to - from);
+        if (to == nb) break;
+        __syncthreads();
     }
-    if (!totals) return;
-    __syncthreads();
-    const uint32_t t = threadIdx.x;
-    if (t < 4u && first + t < placed) totals[first + t] = ordered_total(block_sums + t * nb, nb);
+    if (t < 4u && first + t < placed) totals[first + t] = total;
 }
 
 // GLM's profile: each placed row-slot's down finish as f32 [row-slot][hidden] (routed_slots_block's statements), by
@@ -834,6 +869,32 @@ hipError_t launch_gemm(const PfGemm& g, int codebook, uint32_t max_items, uint32
     });
 }
 
+template <bool TOTALS>
+hipError_t launch_pf_prep(const MoeLaunch& a, hipStream_t s) {
+    const uint32_t p = a.rows * (a.topk + a.shared_slots), nb = a.hidden / 128u, groups = (p + 3u) / 4u;
+    const uint32_t want = stage_waves(p, nb, TOTALS), y = (want + 3u) / 4u, parts = TOTALS ? want : 4u * y;
+    const dim3 grid(groups, TOTALS ? 1u : y), block(TOTALS ? 64u * parts : 256u);
+    const size_t lds = TOTALS ? parts * 1024u + 2u * sum_chunk(nb) * 16u : 4096u;
+    float* totals = TOTALS ? a.xt : nullptr;
+    if (!TOTALS && a.glm) hipLaunchKernelGGL((pf_prep<kBf16, 1, false>), grid, block, lds, s, a, totals, p, parts);
+    else if (a.dtype == kF32) hipLaunchKernelGGL((pf_prep<kF32, 0, TOTALS>), grid, block, lds, s, a, totals, p, parts);
+    else if (a.dtype == kF16) hipLaunchKernelGGL((pf_prep<kF16, 0, TOTALS>), grid, block, lds, s, a, totals, p, parts);
+    else hipLaunchKernelGGL((pf_prep<kBf16, 0, TOTALS>), grid, block, lds, s, a, totals, p, parts);
+    return hipGetLastError();
+}
+
+template <bool TOTALS>
+hipError_t launch_pf_mid(const MoeLaunch& a, hipStream_t s) {
+    const uint32_t p = a.rows * (a.topk + a.shared_slots), nb = a.inter / 128u, groups = (p + 3u) / 4u;
+    const uint32_t parts = stage_waves(p, nb, TOTALS);
+    const dim3 grid = TOTALS ? dim3(groups) : dim3((groups + 3u) / 4u, parts), block(TOTALS ? 64u * parts : 256u);
+    const size_t lds = TOTALS ? parts * 1024u + sum_chunk(nb) * 16u : 4096u;
+    float* totals = TOTALS ? a.xt + 2u * static_cast<size_t>(p) : nullptr;
+    if (!TOTALS && a.glm) hipLaunchKernelGGL((pf_mid<1, false>), grid, block, lds, s, a, totals, parts);
+    else hipLaunchKernelGGL((pf_mid<0, TOTALS>), grid, block, lds, s, a, totals, parts);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 bool dense_prefill_pairs(const DenseLaunch& d) {
@@ -856,14 +917,9 @@ hipError_t launch_moe_prefill(const MoeLaunch& a, hipStream_t s) {
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (a.stages & 2u) {
-        float* totals = map ? a.xt : nullptr;
-        const dim3 grid = position_grid(p), block(256);
-        const size_t sums = map ? 8u * (a.hidden / 128u) * 4u : 0u;
-        if (a.glm) hipLaunchKernelGGL((pf_prep<kBf16, 1>), grid, block, sums, s, a, totals, p);
-        else if (a.dtype == kF32) hipLaunchKernelGGL((pf_prep<kF32, 0>), grid, block, sums, s, a, totals, p);
-        else if (a.dtype == kF16) hipLaunchKernelGGL((pf_prep<kF16, 0>), grid, block, sums, s, a, totals, p);
-        else hipLaunchKernelGGL((pf_prep<kBf16, 0>), grid, block, sums, s, a, totals, p);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (map) e = launch_pf_prep<true>(a, s);
+        else e = launch_pf_prep<false>(a, s);
+        if (e != hipSuccess) return e;
     }
 
     PfGemm g{};
@@ -891,11 +947,9 @@ hipError_t launch_moe_prefill(const MoeLaunch& a, hipStream_t s) {
     }
 
     if (a.stages & 8u) {
-        float* totals = map ? a.xt + 2u * static_cast<size_t>(p) : nullptr;
-        const size_t sums = map ? 4u * (a.inter / 128u) * 4u : 0u;
-        if (a.glm) hipLaunchKernelGGL(pf_mid<1>, position_grid(p), dim3(256), sums, s, a, totals);
-        else hipLaunchKernelGGL(pf_mid<0>, position_grid(p), dim3(256), sums, s, a, totals);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (map) e = launch_pf_mid<true>(a, s);
+        else e = launch_pf_mid<false>(a, s);
+        if (e != hipSuccess) return e;
     }
 
     g.w[0] = a.bank.down_t;
