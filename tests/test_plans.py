@@ -99,8 +99,10 @@ def test_few_rows_share_the_tile_rows_out(lib):
     assert (w.path, w.launches, w.k_slices) == (4, 3, 1)
     assert [linear_plan(lib, r, 4096, 14336, 64, BF16).path for r in (512, 513)] == [3, 4]
     assert [linear_plan(lib, r, 7168, 2048, 48, BF16).path for r in (512, 1024, 4096)] == [3, 4, 4]
-    few = linear_plan(lib, 1024, 7168, 2048, 48, BF16)      # 4 x 8 tiles: eight K parts of 28 steps fill the 256 compute units
-    assert (few.k_slices, few.launches, few.workgroups) == (8, 4, 256)
+    # 7168 x 2048 at 1024 rows: 8 x 8 tiles of 128 rows in four K parts of 56 steps (57 us a call; four times eight 256-row tiles in
+    # eight parts of 28 steps fill the compute units as well and pay for twice the planes: 65)
+    few = linear_plan(lib, 1024, 7168, 2048, 48, BF16)
+    assert (few.k_slices, few.launches, few.workgroups) == (4, 4, 256)
     cfg = Config()
     lib.t3_config_default(C.byref(cfg))
     cfg.dense_gemm_rows = 0
@@ -110,6 +112,22 @@ def test_few_rows_share_the_tile_rows_out(lib):
     finally:
         lib.t3_config_default(C.byref(cfg))
         assert lib.t3_configure(C.byref(cfg)) == 0
+
+
+@pytest.mark.parametrize("in_f,out_f", [(1024, 4096), (4096, 1024), (4096, 2048), (8192, 1024), (8192, 2048), (7168, 2048),
+                                        (4096, 14336), (14336, 4096), (640, 128)])
+def test_the_w_hat_plan_adds_up(lib, in_f, out_f):
+    # whole K parts of eight steps (K = 32) or more, inside one round of the 256 compute units; the finish is a launch of its own
+    # where there are parts
+    for rows in (513, 600, 768, 1024, 1400, 2048, 4096):
+        p = linear_plan(lib, rows, in_f, out_f, 64, BF16)
+        assert (p.path, p.launches) == (4, 3 if p.k_slices == 1 else 4)
+        columns = (out_f + 255) // 256
+        assert p.workgroups % (columns * p.k_slices) == 0
+        tile_rows = [t for t in (64, 96, 128, 192, 256) if (rows + t - 1) // t * columns * p.k_slices == p.workgroups]
+        assert tile_rows, p.workgroups
+        if p.k_slices > 1:
+            assert p.workgroups <= 256 and in_f // 32 % p.k_slices == 0 and in_f // 32 // p.k_slices >= 8
 
 
 def test_config3_routed_partition(lib):

@@ -266,14 +266,11 @@ inline GemmShape gemm_shape(uint32_t rows, uint32_t in, uint32_t cols, bool plan
     }
     return best;
 }
-// The W_hat form's shape. Where 256-row tiles are few (32 at most, shared out in eight parts or more) it keeps them and their
-// parts: the plan that t3_linear_plan_of has always published for such calls (7168 x 2048 at 1024 rows: 47 us against 40).
-inline GemmShape w_hat_shape(uint32_t rows, uint32_t in, uint32_t out) {
-    const uint32_t tiles = ((rows + 255u) / 256u) * ((out + 255u) / 256u), steps = in / 32u;
-    uint32_t k = 1;
-    while (k < 16u && tiles * 2u * k <= 256u && steps % (2u * k) == 0u && steps / (2u * k) >= 16u) k *= 2u;
-    return k >= 8u ? GemmShape{256u, k} : gemm_shape(rows, in, out, true);
-}
+// The W_hat form's. (256-row tiles in the parts that fill the GPU, the shape of its calls over few tiles before this rule, against
+// it, us a call: 7168 x 2048 at 600 / 1024 rows 54.6 / 65.4 -> 46.4 / 57.0, 4096 x 2048 at 513 / 1024 rows 42.9 / 51.5 -> 34.1 /
+// 42.6, 8192 x 1024 at 513 / 2048 rows 60.5 / 105 -> 47.3 / 91.6; 4096 x 1024 at 600 / 1024 / 2048 rows 37.5 / 43.0 / 72.8 ->
+// 36.5 / 43.7 / 58.2.)
+inline GemmShape w_hat_shape(uint32_t rows, uint32_t in, uint32_t out) { return gemm_shape(rows, in, out, true); }
 inline bool gemm_half_ok(uint64_t in, uint64_t ldw) {
     return in % 32u == 0u && ldw % 8u == 0u && in * ldw * 2u < (1ull << 32);
 }

@@ -101,12 +101,14 @@ uint32_t gemv_rows_max() { return config().dense_rows_alone ? 16u : kGemvRowsMax
 
 // From dense_gemm_rows rows up a dense call decodes W_hat once and multiplies plainly (src/core/dense.zig:909-922,
 // 1290-1302): the decode is paid once a call, not once a 128-row item, and the plain GEMM shares K out where its tiles are
-// few (w_hat_shape), so it fills the GPU at any shape. Measured over ten model shapes x eight row counts from 256 to 4096
-// (trellis GEMM against W_hat form, us): up to 512 rows (four items) the trellis GEMM wins or ties everywhere (4096 x 4096
-// 47 / 63, 4096 x 14336 98 / 109); from five items on the W_hat form does (640 rows: 4096 x 4096 64 / 56, 4096 x 14336
-// 158 / 130, 14336 x 4096 159 / 133, 7168 x 2048 60 / 55; 2048 rows: 2560 x 5120 109 / 84, 8192 x 8192 321 / 270), with
-// ties at 1024 rows and two cells the other way (2048 x 2048 at 2048 rows 49 / 57, 7168 x 2048 at 1024 rows 65 / 75).
-// Hence the default of 513.
+// few (w_hat_shape). Measured over ten weights x fourteen row counts from 128 to 2048 at K4 (trellis GEMM against W_hat form, us
+// a call): up to 512 rows (four items) the trellis GEMM wins at most weights (512 rows: 4096 x 4096 41 / 44, 14336 x 4096 87 /
+// 113, 7168 x 2048 39 / 43; not 4096 x 14336 92 / 86 and, from 300 rows on, 1024 x 4096 26 / 23); from five items on the W_hat
+// form does over weights of 2048 columns and more (513 rows: 4096 x 4096 52 / 49, 4096 x 14336 143 / 105, 14336 x 4096 133 / 117,
+// 4096 x 2048 36 / 34; 2048 rows: 101 / 82, 310 / 249, 288 / 262, 63 / 59), with a tie or two (7168 x 2048 at 513 rows 48 / 48,
+// 14336 x 4096 at 1024 rows 158 / 162). Over 1024 columns the trellis GEMM stays ahead at every row count (4096 x 1024 at 600 /
+// 2048 rows 30 / 37 and 44 / 58, 8192 x 1024 39 / 49 and 67 / 92): the switch is a row count, the caller's to set, and 513 is
+// its default for the widths that a model's projections mostly have.
 bool takes_w_hat(const DenseLaunch& l) {
     const int32_t from = config().dense_gemm_rows;
     return !config().dense_rows_alone && from > 0 && l.rows >= static_cast<uint32_t>(from) && gemm_half_ok(l.in, l.out);
