@@ -96,3 +96,22 @@ def test_hand_written_wide_stores_keep_their_wait_states():
                 found += 1
                 assert re.search(r"_store_\w+[^\"]*\\n\\ts_nop [1-9]", body), f"{name}: a wide store without wait states behind it"
     assert found >= 1  # store_coherent4 (t3_common.hpp)
+
+
+def test_hand_written_sub_dword_adds_keep_their_wait_states():
+    """A sub-dword write wants one wait state before an instruction that keeps the register's other half. In every `asm`
+    statement the add that starts a register is followed by an instruction that leaves that register alone."""
+    text = open(os.path.join(ROOT, "turboexl3_amd", "csrc", "t3_decode.hpp")).read()
+    found = 0
+    for m in re.finditer(r'\basm\(((?:\s*"[^"]*")+)', text):
+        lines = [l.strip() for l in "".join(re.findall(r'"([^"]*)"', m.group(1))).split("\\n\\t")]
+        if "v_add_f16_sdwa" not in lines[0]:
+            continue
+        dest = [re.match(r"v_add_f16_sdwa (%\d+)", l) for l in lines]
+        for i, line in enumerate(lines):
+            if "dst_sel:WORD_0" not in line:
+                continue
+            found += 1
+            assert i + 1 < len(lines), f"nothing behind {line}"
+            assert dest[i + 1] is None or dest[i + 1].group(1) != dest[i].group(1), f"{line} and {lines[i + 1]} touch one register"
+    assert found == 3  # weight_halves8: two registers a block, or one

@@ -699,3 +699,35 @@ def test_glm_profile_slots_against_float64(oracle, t3, hidden, inter, experts, r
             assert q <= 1.0, f"rows {rows} row {r} slot {j}: {q:.3f} of its tolerance"
             worst = max(worst, q)
     print(f"GLM profile hidden {hidden} rows {rows}: worst {worst:.3f} of the float64 tolerance")
+
+
+@pytest.mark.parametrize("codebook", [MCG, MUL1])
+@pytest.mark.parametrize("n", [16, 36, 48, 64, 72, 80, 100, 128])
+@pytest.mark.parametrize("wbits", [16, 11])
+def test_rows_of_a_many_row_call_equal_their_own_calls(t3, n, codebook, wbits):
+    """Calls of up to four rows and calls of more take kernels that decode the same weights with other instructions: nine rows,
+    through the two-launch, the four-launch and the grouped form, against each row alone, byte for byte, at every reader of the
+    codes."""
+    hidden, inter, experts, topk, rows = 512, 384, 24, 3, 9
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + wbits)
+
+    def proj(in_f, out_f):
+        return t3.Proj(torch.randint(-32768, 32768, (experts, in_f // 16, out_f // 16, n), dtype=torch.int16, device="cuda",
+                                     generator=g),
+                       torch.randn(experts, in_f, device="cuda", generator=g).half(),
+                       (torch.randn(experts, out_f, device="cuda", generator=g) * in_f ** -0.5).half())
+
+    bank, dec = t3.Bank(proj(hidden, inter), proj(hidden, inter), proj(inter, hidden)), t3.Decode(codebook, wbits)
+    x = torch.randn(1, rows, hidden, device="cuda", generator=g).bfloat16()
+    inds = torch.rand(rows, experts, device="cuda", generator=g).topk(topk).indices.to(torch.int32)[None].contiguous()
+    scores = torch.rand(1, rows, topk, device="cuda", generator=g)
+    alone = torch.cat([t3.moe(x[:, r:r + 1].contiguous(), bank, inds[:, r:r + 1].contiguous(), scores[:, r:r + 1].contiguous(), dec)
+                       for r in range(rows)], 1)
+    assert bool(torch.isfinite(alone).all()) and float(alone.float().abs().max()) > 0
+    for form in (9, 8, 5):
+        t3.configure(decode_form=form)
+        try:
+            assert bytes_of(t3.moe(x, bank, inds, scores, dec)) == bytes_of(alone), form
+        finally:
+            t3.configure()

@@ -39,19 +39,37 @@ constexpr uint32_t kMul1Mult = 0x83DCD12Du;
 //   1.8-1.9  v_alignbit, v_bfe, v_mul_lo_u32 (and v_mul_u32_u24: no split over the 24-bit multiplier pays), v_sad_u8,
 //            sub-dword adds; v_bitop3 and the plain operations above with a scalar register among their operands, v_bitop3
 //            with its second and third operand of one parity
-// So the constants of a kernel's inner loop sit in vector registers, MCG's two in an aligned pair (neighbours differ in
-// parity), and a window that ends where its register ends is cut with an and. A lane's quad of MCG weights, 17 operations
-// in a row: 27.4 -> 26.4 ns of a SIMD at four waves, 36.5 -> 31.6 at one.
+// So where a kernel's waves are few the constants of its inner loop sit in vector registers, MCG's two in an aligned pair
+// (neighbours differ in parity), and a window that ends where its register ends is cut with an and. A lane's quad of MCG
+// weights, 17 operations in a row: 27.4 -> 26.4 ns of a SIMD at four waves, 36.5 -> 31.6 at one.
 struct DecodeConsts {
+    static constexpr bool kLean = false;
     uint2v mcg;     // the hash's mask, then its exclusive or
     uint32_t mask;  // a window's bits: (1 << wbits) - 1
 };
-__device__ __forceinline__ DecodeConsts decode_consts(uint32_t wbits) {
-    DecodeConsts c;
-    c.mcg = uint2v{0x8FFF8FFFu, 0x3B603B60u};
-    c.mask = (1u << wbits) - 1u;
-    asm volatile("" : "+v"(c.mcg), "+v"(c.mask));  // in vector registers, their values unknown to the compiler
-    return c;
+// Where a launch's waves are many, its kernel keeps no constants: their three registers are a wave of occupancy for the routed
+// GEMVs at four tiles a load (96 registers are five waves a SIMD, 98 four; 78 six, 81 five), and the adds of two weights stand by
+// themselves, between other weights' operations, instead of four to a block. The other form against this one, us a routed call on
+// one box: 512 experts of 2048 x 512 top-10 K3 with a shared expert at 8 / 16 rows 55.0 / 95.2 -> 53.5 / 92.7, 512 of 2560 x 640
+// K4 at 8 rows 84.4 -> 82.0, 64 of 4096 x 1024 top-8 K5 at 4 / 8 rows 89.5 / 128.5 -> 85.1 / 120.8, K8 at 8 rows 143.0 -> 134.6,
+// 256 of 7168 x 2048 K3 at 1 / 2 rows 72.3 / 126.6 -> 70.8 / 123.7. With few waves the other form is the faster: one row of the
+// first 19.98 against 20.10, of the K5 bank 31.9 against 33.1, one dense row of 4096 x 12288 K3 12.08 against 12.23, of
+// 2048 x 2048 6.28 against 6.43.
+struct LeanConsts {
+    static constexpr bool kLean = true;
+};
+template <bool LEAN = false>
+__device__ __forceinline__ auto decode_consts(uint32_t wbits) {
+    if constexpr (LEAN) {
+        (void)wbits;
+        return LeanConsts{};
+    } else {
+        DecodeConsts c;
+        c.mcg = uint2v{0x8FFF8FFFu, 0x3B603B60u};
+        c.mask = (1u << wbits) - 1u;
+        asm volatile("" : "+v"(c.mcg), "+v"(c.mask));  // in vector registers, their values unknown to the compiler
+        return c;
+    }
 }
 
 // cw times a 32-bit constant, modulo 2^32
@@ -74,6 +92,8 @@ __device__ __forceinline__ uint32_t mcg_pair(uint32_t cw, const DecodeConsts& k)
     // (a builtin, not an asm statement: the compiler keeps the wait states before a matrix instruction reads its result)
     return __builtin_amdgcn_bitop3_b32(hash_mul<kMcgMult>(cw), k.mcg[0], k.mcg[1], 0x6A);
 }
+
+__device__ __forceinline__ uint32_t mcg_pair(uint32_t cw, const LeanConsts&) { return mcg_pair(cw); }
 
 // Exact decoders (format.zig:149-167). MCG: both halves have exponents in [2^-3, 2^0], so their f32 sum is exact and
 // one f16 add rounds as f16(f32(lo) + f32(hi)) does. MUL1: (1024 + t) A + B is a multiple of 2^-18 below 4, exact in
@@ -98,8 +118,8 @@ __device__ __forceinline__ uint16_t decode_exact(uint32_t cw) {
 
 // A weight as the GEMV's matrix core takes it where a quad fills the fragment: 32 bits = two f16 K slots (the second zero
 // unless kMcgPair).
-template <int CB>
-__device__ __forceinline__ uint32_t weight_pair(uint32_t cw, const DecodeConsts& k) {
+template <int CB, typename Consts>
+__device__ __forceinline__ uint32_t weight_pair(uint32_t cw, const Consts& k) {
     if constexpr (CB == kMcgPair) return mcg_pair(cw, k);
     else if constexpr (CB == kMul1Defer) return mul1_h(cw);
     else return static_cast<uint32_t>(decode_exact<CB>(cw));
@@ -107,25 +127,46 @@ __device__ __forceinline__ uint32_t weight_pair(uint32_t cw, const DecodeConsts&
 
 // Eight weights as an A fragment's eight f16 K slots: c0's four, then c1's. Exact, or MUL1's h = 1024 + t where its map is
 // deferred.
-template <int CB>
-__device__ __forceinline__ uint4v weight_halves8(const uint32_t (&c0)[4], const uint32_t (&c1)[4], const DecodeConsts& k) {
+template <int CB, typename Consts>
+__device__ __forceinline__ uint4v weight_halves8(const uint32_t (&c0)[4], const uint32_t (&c1)[4], const Consts& k) {
     uint4v a;
     if constexpr (CB == kMcg) {
         // A weight is one f16 add of its hashed pair's halves, and the sub-dword forms of v_add_f16 write the low half,
         // then the high half of the same register. A sub-dword write wants one wait state before the add that keeps it
-        // (two registers' adds take turns) and two before a matrix instruction reads it (the s_nop at the end); the
-        // compiler adds them for its own sub-dword instructions, not for these.
-        auto two = [&](uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t& lo, uint32_t& hi) {
-            asm("v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-                "v_add_f16_sdwa %1, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-                "v_add_f16_sdwa %0, %3, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
-                "v_add_f16_sdwa %1, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
-                : "=&v"(lo), "=&v"(hi)
-                : "v"(mcg_pair(w0, k)), "v"(mcg_pair(w1, k)), "v"(mcg_pair(w2, k)), "v"(mcg_pair(w3, k)));
-        };
+        // (two registers' adds take turns, or an s_nop) and two before a matrix instruction reads it (the s_nop at the
+        // end); the compiler adds them for its own sub-dword instructions, not for these.
         uint32_t r[4];
-        two(c0[0], c0[1], c0[2], c0[3], r[0], r[1]);
-        two(c1[0], c1[1], c1[2], c1[3], r[2], r[3]);
+        if constexpr (Consts::kLean) {
+            // a wait state behind every add: other waves issue in it (without the second one the routed launches of
+            // eight rows measured 1 to 2 % longer)
+            auto two = [&](uint32_t w0, uint32_t w1) {
+                uint32_t d;
+                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+                    "s_nop 0"
+                    : "=v"(d)
+                    : "v"(mcg_pair(w0, k)));
+                asm("v_add_f16_sdwa %0, %1, %1 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+                    "s_nop 0"
+                    : "+v"(d)
+                    : "v"(mcg_pair(w1, k)));
+                return d;
+            };
+            r[0] = two(c0[0], c0[1]);
+            r[1] = two(c0[2], c0[3]);
+            r[2] = two(c1[0], c1[1]);
+            r[3] = two(c1[2], c1[3]);
+        } else {
+            auto two = [&](uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t& lo, uint32_t& hi) {
+                asm("v_add_f16_sdwa %0, %2, %2 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+                    "v_add_f16_sdwa %1, %4, %4 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+                    "v_add_f16_sdwa %0, %3, %3 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+                    "v_add_f16_sdwa %1, %5, %5 dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1"
+                    : "=&v"(lo), "=&v"(hi)
+                    : "v"(mcg_pair(w0, k)), "v"(mcg_pair(w1, k)), "v"(mcg_pair(w2, k)), "v"(mcg_pair(w3, k)));
+            };
+            two(c0[0], c0[1], c0[2], c0[3], r[0], r[1]);
+            two(c1[0], c1[1], c1[2], c1[3], r[2], r[3]);
+        }
         a = uint4v{r[0], r[1], r[2], r[3]};
         asm("s_nop 1" : "+v"(a));
     } else {
@@ -259,18 +300,22 @@ __device__ __forceinline__ QuadWords<WIDE> quad_load(const uint32_t* tile, const
 }
 
 // The quad's four codewords, masked to the pack's window width `wbits` (8..16). The last window of each register ends at its
-// bit 0 (o[3] = 0, and o[1] = 0 of the wide readers): an and where the others take a v_bfe.
-template <int WIDE>
+// bit 0 (o[3] = 0, and o[1] = 0 of the wide readers): an and where the others take a v_bfe, if its mask is in a register.
+template <int WIDE, typename Consts>
 __device__ __forceinline__ void quad_codewords(const QuadWords<WIDE>& w, const QuadPlan<WIDE>& q, uint32_t wbits,
-                                               const DecodeConsts& k, uint32_t (&cw)[4]) {
+                                               const Consts& k, uint32_t (&cw)[4]) {
+    const auto last = [&](uint32_t r) -> uint32_t {
+        if constexpr (Consts::kLean) return __builtin_amdgcn_ubfe(r, 0u, wbits);
+        else return r & k.mask;
+    };
     const uint32_t rb = __builtin_amdgcn_alignbit(w.b_prev, w.b_last, q.shb);
     uint32_t ra = rb;
     if constexpr (WIDE == kWide) ra = __builtin_amdgcn_alignbit(w.a_prev, w.a_last, q.sha);
     if constexpr (WIDE == kWidePair) ra = __builtin_amdgcn_alignbit(w.b_prev, q.a_low ? w.b_prev : w.b_last, q.sha);
     cw[0] = __builtin_amdgcn_ubfe(ra, q.o[0], wbits);
-    cw[1] = WIDE == kNarrow ? __builtin_amdgcn_ubfe(ra, q.o[1], wbits) : ra & k.mask;
+    cw[1] = WIDE == kNarrow ? __builtin_amdgcn_ubfe(ra, q.o[1], wbits) : last(ra);
     cw[2] = __builtin_amdgcn_ubfe(rb, q.o[2], wbits);
-    cw[3] = rb & k.mask;
+    cw[3] = last(rb);
 }
 
 // Tile row of a quad's weight m, and its column: the inverse of the permutation for one lane.

@@ -134,7 +134,8 @@ struct GemvStep {
                 }
             }
     }
-    __device__ __forceinline__ void consume(const QuadPlan<WIDE>& plan, uint32_t wbits, const DecodeConsts& k,
+    template <typename Consts>
+    __device__ __forceinline__ void consume(const QuadPlan<WIDE>& plan, uint32_t wbits, const Consts& k,
                                             const uint4v (&xv)[RB], float4v (&acc)[RB][BT]) const {
 #pragma unroll
         for (int t = 0; t < BT; ++t) {
@@ -158,7 +159,7 @@ struct GemvStep {
     }
 };
 
-template <int CB, int WIDE, int RB, int BT, typename XSrc>
+template <int CB, int WIDE, int RB, int BT, typename XSrc, bool LEAN>
 struct GemvStreamRegs {
     static constexpr int R = gemv_step_rows<CB>();   // tile rows a step
 #ifndef T3_GEMV_REGS_ST2
@@ -247,7 +248,7 @@ struct GemvStreamRegs {
         const uint32_t chunk_bytes = static_cast<uint32_t>(BT) * tile_bytes;
         // The loads are in flight; everything a lane needs to decode is worked out under their latency.
         const QuadPlan<WIDE> plan = quad_plan<WIDE>(n, lane);
-        const DecodeConsts consts = decode_consts(wbits);
+        const auto consts = decode_consts<LEAN>(wbits);
         // where the lane's four loaded dwords land: tile slot + offset inside the tile (a lane past the chunk stores
         // into the dump behind the buffers); b / tile_bytes by a 16-bit reciprocal, exact for b < 1024 and
         // tile_bytes >= 32
@@ -342,7 +343,7 @@ struct GemvStreamRegs {
     }
 };
 
-template <int CB, int WIDE, int RB, int BT, typename XSrc>
+template <int CB, int WIDE, int RB, int BT, typename XSrc, bool LEAN>
 struct GemvStreamLds {
 #ifndef T3_GEMV_LDS_RING_DEPTH
 #define T3_GEMV_LDS_RING_DEPTH 4
@@ -407,7 +408,7 @@ struct GemvStreamLds {
     __device__ __forceinline__ void run(float4v (&acc)[RB][BT]) {
         // The loads are in flight; everything a lane needs to decode is worked out under their latency.
         const QuadPlan<WIDE> plan = quad_plan<WIDE>(n, lane);
-        const DecodeConsts consts = decode_consts(wbits);
+        const auto consts = decode_consts<LEAN>(wbits);
         // a step's activations: the LDS form's out of the wave's prepared block (past the last: the zero step), the
         // others out of the register ring
         auto fetch_x = [&](int slot, uint32_t step, uint4v(&xv)[RB]) {
@@ -479,8 +480,9 @@ struct GemvStreamLds {
     }
 };
 
-// LDS: the direct-to-LDS ring; else the register ring
-template <bool LDS, int CB, int WIDE, int RB, int BT, typename XSrc>
-using GemvStream = std::conditional_t<LDS, GemvStreamLds<CB, WIDE, RB, BT, XSrc>, GemvStreamRegs<CB, WIDE, RB, BT, XSrc>>;
+// LDS: the direct-to-LDS ring; else the register ring. LEAN: the decode of launches of many waves (LeanConsts).
+template <bool LDS, int CB, int WIDE, int RB, int BT, typename XSrc, bool LEAN = false>
+using GemvStream =
+    std::conditional_t<LDS, GemvStreamLds<CB, WIDE, RB, BT, XSrc, LEAN>, GemvStreamRegs<CB, WIDE, RB, BT, XSrc, LEAN>>;
 
 }  // namespace t3

@@ -72,8 +72,11 @@ template <int CB, int WIDE, int BT, int NPROJ, bool XLDS, bool ARRIVE, int PROF,
 __device__ __forceinline__ void gemv_role(const MoeLaunch& a, uint32_t blk, uint32_t yidx, uint32_t ksl,
                                           unsigned char* smem, unsigned char* xbase, uint32_t& last_flag, uint32_t* cinfo,
                                           float* cscore) {
-    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XLds> StreamL;
-    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XGlobal> StreamG;
+    // few waves: the launches of calls of up to four rows, which make their own inputs and, gate|up, leave the planes to the down
+    // launch; but not gate|up at eight tiles a load, which those calls take where it has more than 2048 workgroups
+    constexpr bool kLean = NPROJ == 1 ? !XLDS : !XLDS || ARRIVE || BT == 8;
+    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XLds, kLean> StreamL;
+    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XGlobal, kLean> StreamG;
     constexpr uint32_t kStage = StreamG::kStageBytes;
     static_assert(kStage <= role_wave_lds_bytes<BT>() && StreamL::kStageBytes <= role_wave_lds_bytes<BT>(), "a wave's ring fits its share");
     constexpr int R = gemv_step_rows<CB>();   // tile rows a step
@@ -475,7 +478,7 @@ constexpr uint32_t group_lds_bytes() {
 template <int CB, int WIDE, int BT, int NPROJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : (gemv_step_rows<CB>() == 2 ? 3 : 4)))) moe_gemv_grouped(const MoeLaunch a) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[group_lds_bytes<BT>()];
-    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XGlobal> StreamG;
+    typedef GemvStream<kMoeLdsRing, CB, WIDE, 1, BT, XGlobal, true> StreamG;
     constexpr uint32_t kStage = StreamG::kStageBytes;
     const uint32_t g = blockIdx.y / NPROJ, proj = blockIdx.y % NPROJ, blk = blockIdx.x, ksl = blockIdx.z;
     if (g >= a.groups[0]) return;  // uniform over the workgroup
