@@ -88,7 +88,10 @@ def _compile_torch(force: bool) -> str:
 
     obj = os.path.join(OBJDIR, "t3_torch.cpp.o")
     path = os.path.join(CSRC, "t3_torch.cpp")
-    if not force and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(path), _headers_mtime()):
+    # the torch and the Python it was built for: file times say nothing of another one in their place
+    built_for, stamp = f"{torch.__version__} {torch.__file__} {sys.version}", obj + ".built_for"
+    same = os.path.exists(stamp) and open(stamp).read() == built_for
+    if not force and same and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(path), _headers_mtime()):
         return obj
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
     includes = [inc, os.path.join(inc, "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
@@ -97,6 +100,8 @@ def _compile_torch(force: bool) -> str:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("g++ failed on t3_torch.cpp:\n" + res.stderr)
+    with open(stamp, "w") as f:
+        f.write(built_for)
     return obj
 
 
