@@ -227,11 +227,11 @@ int32_t admit_prefill(const MoeCall& call) {
 // The two launches save three launch boundaries (~12 us of the chain) and pay with every gate|up workgroup's own prepare
 // of its block (once a column workgroup instead of once) and the coherent hand-offs, ~8 % of the decode at eight tiles a
 // load and twice that at four: past eight rounds of the GPU's resident workgroups the five launches are faster. Measured
-// (two against five, us): 4096 x 2048 K4 top-8 at 4 / 5 / 8 / 16 rows 148.7 / 177.0 / 270.8 / 515.5 against 148.5 / 175.3 /
-// 256.1 / 477.5; 7168 x 2048 K3 at 2 / 3 / 8 rows 131.9 / 189.0 / 449.4 against 133.9 / 180.1 / 415.6; 4096 x 1024 K5 at
-// 4 / 8 rows 96.6 / 170.9 against 95.7 / 159.2; 2048 x 512 K3 top-10 at 16 rows 97.1 against 103.1. Past the bound the decode
-// is what the call waits for, and serving the row-slots of one expert together pays (five against grouped, us: 4096 x 2048
-// top-8 of 64 at 8 / 16 rows 256 / 468 against 208 / 274; eight experts of 4096 x 14336 top-2 at 16 rows 754 against 254).
+// (two against five, us): 4096 x 2048 K4 top-8 at 3 / 4 / 5 / 8 / 16 rows 110.6 / 141.3 / 156.9 / 237.3 / 449.9 against 110.5 /
+// 135.8 / 161.3 / 235.8 / 433.6; 7168 x 2048 K3 at 2 / 3 / 8 rows 126.1 / 180.6 / 410.9 against 124.4 / 170.1 / 397.3; 4096 x 1024
+// K5 at 4 / 8 rows 89.7 / 146.3 against 84.6 / 140.1; 2048 x 512 K3 top-10 at 16 rows 92.1 against 102.7. Past the bound the
+// decode is what the call waits for, and serving the row-slots of one expert together pays (five against grouped, us: 4096 x 2048
+// top-8 of 64 at 8 / 16 rows 236 / 434 against 178 / 238; eight experts of 4096 x 4096 top-2 at 16 rows 207 against 78).
 // Every form gives the same bytes, so a row's bytes do not depend on which one its call took.
 constexpr uint64_t kTwoLaunchGroups = 8192u;
 int decode_form_of(const MoeLaunch& l) {
@@ -250,9 +250,10 @@ int decode_form_of(const MoeLaunch& l) {
     // Below the bound the six launches cost ~20 us more of chain than the two, and win where grouping removes more decode
     // than that: by the groups a uniform routing is expected to leave (E (1 - (1 - k / E)^rows) experts hit, one group a
     // shared slot), gate|up workgroups saved = gu_groups (1 - groups / row-slots). Measured crossover ~1400 (two against
-    // grouped, us: 128 experts of 2048 x 768 top-8 at 16 rows, 2200 saved, 108 / 96; 16 experts of 2048 x 1024 top-4 at 16
-    // rows, 3100 saved, 68 / 49, at 8 rows, 1100 saved, 43 / 43; 512 of 2048 x 512 top-10 + shared at 16 rows, 1200 saved,
-    // 100 / 106). A skewed routing groups better than this estimate.
+    // grouped, us: 128 experts of 2048 x 768 top-8 at 12 rows, 1300 saved, 82.3 / 83.4, at 16 rows, 2200 saved, 102.8 / 93.3;
+    // 16 experts of 2048 x 1024 top-4 at 8 rows, 1100 saved, 39.4 / 41.7, at 12 rows, 2100 saved, 53.4 / 43.7; 512 of 2048 x 512
+    // top-10 + shared at 16 rows, 1200 saved, 92 / 102; the other way 8 experts of 4096 x 4096 top-2 at 4 rows, 1300 saved, 71 /
+    // 61: its down launch, which the estimate leaves out, saves as much). A skewed routing groups better than this estimate.
     if (l.rows >= 2u) {
         const double e = static_cast<double>(l.bank.experts), k = static_cast<double>(l.topk);
         const double hit = e * (1.0 - __builtin_pow(1.0 - (k < e ? k / e : 1.0), static_cast<double>(l.rows)));

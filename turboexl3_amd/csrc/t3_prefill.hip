@@ -830,15 +830,9 @@ hipError_t launch_pf_dense_finish(const DenseLaunch& d, const float* z, bool pai
     return hipGetLastError();
 }
 
-// workgroup columns of a GEMM over `out` columns with `item_rows`-row items
-inline uint32_t gemm_nblk(uint32_t out, uint32_t item_rows) {
-    (void)item_rows;
-    return (out + 255u) / 256u;
-}
-
 template <int CB, int WIDE>
 hipError_t launch_gemm_rb(PfGemm g, uint32_t max_items, uint32_t nproj, uint32_t item_rows, hipStream_t s) {
-    g.nblk = gemm_nblk(g.out, item_rows);
+    g.nblk = (g.out + 255u) / 256u;
     g.spread = gemm_spread(max_items);  // 8 / spread items share the dies
     if (g.kparts == 0u) g.kparts = 1u;
     if constexpr (CB != kMul1) {
