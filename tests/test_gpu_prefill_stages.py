@@ -90,3 +90,32 @@ def test_block_sums_of_very_wide_rows(hidden, inter):
     step = 2.0 ** -10
     worst = ((y[:, :4] - want).abs() - 3 * step * want.abs()).div(5 * 6 ** 0.5 * step * rms).max()
     assert float(worst) <= 1.0, float(worst)
+
+
+@pytest.mark.parametrize("hidden,inter", [(1152, 1408), (1408, 384), (2176, 1152)])
+@pytest.mark.parametrize("decode", ["mcg", "mul1"])
+@pytest.mark.parametrize("rows,topk", [(18, 2), (150, 5)])
+def test_rows_within_the_roundings_of_their_decode_calls(hidden, inter, decode, rows, topk):
+    """Nine to seventeen 128-blocks a position, skipped slots among them, scales with full mantissas: f16 rows against the
+    decode chain, which rounds at the same points and adds the sums up in another order."""
+    from turboexl3_amd import api as t3
+    dec = getattr(t3.Decode, decode)
+    x, bank, inds, scores = case(t3, hidden, inter, rows, topk)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    for p in (bank.gate, bank.up, bank.down):  # magnitudes 1 to 2, so that no column's noise is far above the row's
+        for v in (p.suh, p.svh):
+            v.copy_(torch.where(v < 0, -1.0, 1.0) * (1.0 + torch.rand(v.shape, device="cuda", generator=g)) * (v.float().square().mean() ** 0.5))
+    y = t3.moe(x, bank, inds, scores, dec).float()
+    some = list(range(0, rows, max(1, rows // 25)))
+    want = torch.cat([t3.moe(x[:, r:r + 1].contiguous(), bank, inds[:, r:r + 1].contiguous(), scores[:, r:r + 1].contiguous(), dec)
+                      for r in some], 1).float()
+    # A f32 sum of N terms in another order moves by about sqrt(N) 2^-24 of its rms, under MUL1's map 3.5 times that: at most 0.04
+    # of the distance between two f16 roundings (2^-11) for the N here, so at most one value in twenty rounds the other way, by a
+    # step of 2^-10 of it at most. An element's own three roundings move it by three steps; the six of the gate, up and hidden
+    # values come through the transforms and sums as noise of sqrt(6 / 20) steps of the row's rms, twice that in a column of the
+    # largest scale; five times that is the largest of the 60,000 values looked at.
+    step = 2.0 ** -10
+    rms = want.square().mean(-1, keepdim=True).sqrt()
+    worst = ((y[:, some] - want).abs() - 3 * step * want.abs()).div(5 * 2 * (6 / 20) ** 0.5 * step * rms).max()
+    assert float(worst) <= 1.0, float(worst)

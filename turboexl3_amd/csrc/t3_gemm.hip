@@ -16,9 +16,9 @@
 // 43 us), and so did bypassing the first cache level on the way to LDS (333 rows: 63 -> 68).
 //
 // Memory path. Both operands go from memory straight into LDS (buffer_load ... lds: lane L's 16 bytes land at
-// M0 + 16 L), four steps deep, up to 32 KB a step; the kernel counts those loads itself (s_waitcnt vmcnt(N)) and issues no
-// other vector-memory load while they fly. Which global piece a lane fetches decides the LDS layout at 16-byte
-// granularity, so both tiles are swizzled for their readers on the way in, at no cost:
+// M0 + 16 L), four (256-row tiles) to seven (64-row ones) steps deep, 32 to 20 KB a step; the kernel counts those loads
+// itself (s_waitcnt vmcnt(N)) and issues no other vector-memory load while they fly. Which global piece a lane fetches
+// decides the LDS layout at 16-byte granularity, so both tiles are swizzled for their readers on the way in, at no cost:
 //   activations  [tile rows][32 k], 64 bytes a row; the 16-byte piece p of row r sits at position p ^ ((r >> 1) & 3):
 //                a B fragment (16 rows x one piece) then spreads over all banks (ds_read_b128);
 //   weights      [32 k][256 columns] as they lie in memory (k-major), 512 bytes a row; piece s of row k sits at
@@ -34,7 +34,7 @@
 // finish kernel, then y in the call's dtype. z never sees memory.
 // Workgroup ids: consecutive ids go round the eight dies; a die takes column blocks nt = 8 j + die and walks every row
 // block of one column block before the next, so a die's L2 holds the weight strip its workgroups share. A workgroup
-// holds a compute unit alone (80 to 135 KB of LDS), so the launch runs in rounds of 256 workgroups; where the last round of
+// holds a compute unit alone (132 to 144 KB of LDS), so the launch runs in rounds of 256 workgroups; where the last round of
 // 256-row tiles would fill at most half the GPU, its column blocks are cut to 128 columns (the same kernel with two column blocks a wave):
 // 4096 rows x 14336 columns is 896 tiles = 3.5 rounds, and runs as 768 full tiles + 256 half ones.
 
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(512) gemm_half(const GemmArgs a) {
             load_to_lds(wdesc, base + kGXBytes + (2u * wave + i) * 1024u, w_voff[i], at * w_step_bytes);
     };
 
-    // where a lane's fragments sit inside a step's 32 KB
+    // where a lane's fragments sit inside a step's slot of the ring
     // activations, row block rb: row 16 RBN wm + 16 rb + lane % 16, piece lane / 16, swizzled
     const uint32_t xf_at = (16u * RBN * wm + (lane & 15u)) * 64u + (((lane >> 4) ^ ((lane >> 1) & 3u)) * 16u);
     const uint32_t g = lane >> 4, j = lane & 15u;

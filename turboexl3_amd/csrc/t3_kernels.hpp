@@ -188,8 +188,8 @@ inline uint32_t dense_prefill_kparts(uint32_t rows, uint32_t in, uint32_t out) {
 // Whether two of the dense call's d.ks K parts share a workgroup of eight waves, and the planes of z that leaves: the 128-row
 // shape (more than 64 rows) where the parts alone are more than one workgroup a compute unit; not with MUL1's map inside the
 // weights, which no default configuration runs. Up to 256 workgroups a pair would put two parts on one compute unit and leave
-// another idle: 7168 x 2048 at 256 rows 36.3 us paired, 31.8 with the parts apart; 4096 x 4096 at 128 rows 31.2 and 26.8.
-// Above: 4096 x 14336 at 128 / 200 / 512 rows 43.4 / 58.2 / 95.1 -> 36.6 / 49.5 / 86.7, 4096 x 4096 at 200 rows 35.6 -> 28.4.
+// another idle: 7168 x 2048 at 256 rows 34.8 us paired, 31.4 with the parts apart; 4096 x 4096 at 128 rows 31.3 and 27.3.
+// Above: 4096 x 14336 at 128 / 200 / 512 rows 45.5 / 54.8 / 93.4 -> 39.3 / 50.2 / 84.3, 4096 x 4096 at 200 rows 33.7 -> 29.2.
 bool dense_prefill_pairs(const DenseLaunch& d);
 inline uint32_t dense_prefill_planes(const DenseLaunch& d) { return dense_prefill_pairs(d) ? d.ks / 2u : d.ks; }
 

@@ -759,7 +759,7 @@ __global__ void __launch_bounds__(256) pf_dense_prep(const void* x, const uint16
 }
 
 // the dense finish: z f32 [ks][rows][out], the planes summed in part order (pairs: each even plane with the next one first,
-// as the GEMM's workgroups of two parts do, so that a row's sums are the same however many rows the call has), with
+// as the GEMM's workgroups of two parts do: calls of one number of K parts give a row the same sums, paired or not), with
 // xs [rows][in / 128] for MUL1's deferred map. Four planes' loads are in flight at a time.
 template <int DT>
 __global__ void __launch_bounds__(256) pf_dense_finish(const float* z, const float* xs, const uint16_t* svh, void* y,
